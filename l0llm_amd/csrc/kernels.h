@@ -84,6 +84,9 @@ struct GemvParams {
 int gemv_max_blocks(int compute_units, int per_cu = 2);
 
 int launch_gemv_nk(hipStream_t s, const GemvParams& p);
+// Up to 64 fp32 activation rows against int8, fp16 or bf16 weights (rows_kernel.h); the caller has
+// checked sizes and alignment (launch_gemv_nk).
+int launch_gemv_rows(hipStream_t s, const GemvParams& p, int pos0);
 
 // Reference layout [K, N] GEMV / GEMM (Gemv.Execute, Gemm.Execute): rows in groups of up to 8,
 // K split into `splits` slices of `ks` rows whose fp32 partials go to `ws` (the launcher uses
