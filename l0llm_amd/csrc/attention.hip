@@ -30,7 +30,7 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kGroupMax = 8;  // q heads per kv head
-constexpr int kUnroll = 4;    // positions per slot per step
+constexpr int kUnroll = 4;    // positions per slot per step (1 or 2 for slices that short)
 constexpr int kMaxSplits = 256;
 
 // Reduce-scatter of 16 values over a 16-lane row: on return, lane r of the row holds the sum over
@@ -106,8 +106,8 @@ __device__ __forceinline__ void load8(const void* base, size_t idx, float* f) {
 __host__ __device__ constexpr int partial_stride(int G, int HD) { return G * HD + ((2 * G + 3) / 4) * 4; }
 
 // Sequence length of batch entry b, and this split's slice [lo, lo + n) of it. Slices are whole
-// steps (NG * kUnroll positions) so a block's slots stay in step.
-template <int NG>
+// steps (NG * U positions) so a block's slots stay in step.
+template <int NG, int U>
 __device__ __forceinline__ void split_range(const AttnParams& p, int seq_len_step, int b, int split, int& lo, int& n,
                                             int& len) {
     // The device-side length is read unconditionally (from q, then ignored, when the length is a
@@ -118,7 +118,7 @@ __device__ __forceinline__ void split_range(const AttnParams& p, int seq_len_ste
     asm volatile("" : "+s"(dev_len));
     len = (on_device ? dev_len + p.seq_len_add : p.seq_len) + b * seq_len_step;
     len = max(0, min(len, p.max_seq_len));
-    constexpr int kStep = NG * kUnroll;
+    constexpr int kStep = NG * U;
     int chunk = (len + p.splits - 1) / p.splits;
     chunk = (chunk + kStep - 1) / kStep * kStep;
     lo = split * chunk;
@@ -127,19 +127,17 @@ __device__ __forceinline__ void split_range(const AttnParams& p, int seq_len_ste
 
 // QT: q dtype, G: q heads per kv head rounded up to a power of two (heads >= p.nh / p.nkv are
 // computed on clamped inputs and not written). SC: the reduce-scattered softmax where the shape
-// allows it (head_dim 128, four heads per kv head). SHORT: every slice is at most two steps long
-// (the launch checks max_seq_len against the split count).
-template <int HD, int CT, int QT, int G, bool SC = false, bool SHORT = false>
+// allows it (head_dim 128, four heads per kv head). U: positions per slot per step. ST: every slice
+// is at most ST steps long, 1 or 2 (the launch checks max_seq_len against the split count); 0: any.
+template <int HD, int CT, int QT, int G, int U, int ST, bool SC = false>
 __global__ __launch_bounds__(kBlock) void attn_split_kernel(const AttnParams p, int seq_len_step,
                                                             size_t cache_batch_stride) {
     constexpr int LPP = HD / 8;     // lanes per position
     constexpr int PPW = 64 / LPP;   // position slots per wave
     constexpr int NG = kWaves * PPW;  // position slots per block
-    constexpr int U = kUnroll;
     using T = typename CacheRow<CT>::T;
-    constexpr int NSL = NG;  // position slots of the block (kWaves * PPW)
-    __shared__ float s_m[NSL][G], s_l[NSL][G], s_c[NSL][G], s_M[G];
-    __shared__ float s_acc[NSL][G][HD];
+    __shared__ float s_m[kWaves][G], s_l[kWaves][G];
+    __shared__ __attribute__((aligned(16))) float s_acc[kWaves][G * HD];
 
     const int g = blockIdx.x, split = blockIdx.y, b = blockIdx.z;
     const int gsize = p.nh / p.nkv;
@@ -149,7 +147,7 @@ __global__ __launch_bounds__(kBlock) void attn_split_kernel(const AttnParams p, 
     const int lg = lane % LPP;
     const int slot = wave * PPW + lane / LPP;
     int lo, n, len;
-    split_range<NG>(p, seq_len_step, b, split, lo, n, len);
+    split_range<NG, U>(p, seq_len_step, b, split, lo, n, len);
 
     // q: this lane's 8 dims of every head of the group, scaled by log2(e) / sqrt(HD).
     float qr[G][8];
@@ -165,7 +163,7 @@ __global__ __launch_bounds__(kBlock) void attn_split_kernel(const AttnParams p, 
 #pragma unroll
             for (int d = 0; d < 8; d++) qr[h][d] *= qscale;
     };
-    if constexpr (!SHORT) scale_q();
+    if constexpr (ST == 0) scale_q();
     const T* kbase = static_cast<const T*>(p.kc) + (size_t)b * cache_batch_stride + (size_t)g * HD + lg * 8;
     const T* vbase = static_cast<const T*>(p.vc) + (size_t)b * cache_batch_stride + (size_t)g * HD + lg * 8;
     // Positions past the slice read the last written row (masked in the softmax, weight exactly 0),
@@ -320,23 +318,22 @@ __global__ __launch_bounds__(kBlock) void attn_split_kernel(const AttnParams p, 
     };
 
     // Steps of NG * U positions; the next step's rows are requested before the current one is
-    // computed, and the last step is computed with nothing issued behind it. SHORT (slices of at
-    // most two steps, chosen by the launch): straight-line code that requests both steps, with q,
-    // before computing either. The loop below would take two memory round trips in a row there:
+    // computed, and the last step is computed with nothing issued behind it. ST 1 and 2 (slices of
+    // that many steps at most, chosen by the launch): straight-line code that requests all the steps,
+    // with q, before computing any. The loop below would take two memory round trips in a row there:
     // the compiler's copy of the first step's rows into the loop registers waits for all of them
-    // before the second step is requested. A second step past the slice is fully masked (every
-    // weight is exactly 0, no running maximum moves), so computing it changes no bit.
+    // before the second step is requested.
     const int steps = (n + NG * U - 1) / (NG * U);  // block-uniform
-    if constexpr (SHORT) {
+    if constexpr (ST > 0) {
         load(ka, va, 0);
-        load(kb, vb, 1);
+        if constexpr (ST == 2) load(kb, vb, 1);
         // Nothing moves above this point: left alone, the scheduler scales q (waiting for it) before
         // requesting most of the rows.
         __builtin_amdgcn_sched_barrier(0);
         scale_q();
-        if (steps > 0) {
-            compute(ka, va, 0);
-            compute(kb, vb, 1);
+        if (steps > 0) compute(ka, va, 0);
+        if constexpr (ST == 2) {
+            if (steps > 1) compute(kb, vb, 1);
         }
     } else if (steps > 0) {
         load(ka, va, 0);
@@ -369,28 +366,59 @@ __global__ __launch_bounds__(kBlock) void attn_split_kernel(const AttnParams p, 
         }
     }
 
-    // Combine the block's slots through LDS, in a fixed order: every slot's LPP lanes write their 8
-    // dims of every head and its first lane the running maxima and sums; then each (slot, head)
-    // gets its weight 2^(m - M) against the head's block maximum M; then each output (head, dim)
-    // sums its slots' weighted accumulators and sums.
+    // Combine the wave's slots in registers, in a fixed order: each head's maximum M and weighted sum
+    // over the slots, then the accumulators, weighted by 2^(m - M). Those are reduce-scattered over the
+    // four 16-lane rows (a row swap puts the halves that two rows keep side by side, one add reduces
+    // both), which leaves a lane 2 G of its G * 8 sums; slots that share a row are summed by rotations.
+    constexpr int N8 = G * 8, N4 = N8 / 4;
+    float a4[N4];
+    {
+        float f[N8];
 #pragma unroll
-    for (int h = 0; h < G; h++) {
-        float4* dst = reinterpret_cast<float4*>(&s_acc[slot][h][lg * 8]);
-        dst[0] = make_float4(acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
-        dst[1] = make_float4(acc[h][4], acc[h][5], acc[h][6], acc[h][7]);
-        if (lg == 0) {
-            s_m[slot][h] = m[h];
-            s_l[slot][h] = l[h];
+        for (int h = 0; h < G; h++) {
+            const float M = slot_reduce<LPP, true>(m[h]);
+            const float c = M == -INFINITY ? 0.f : exp2_hw(m[h] - M);
+            m[h] = M;
+            l[h] = slot_reduce<LPP, false>(l[h] * c);
+#pragma unroll
+            for (int d = 0; d < 8; d++) f[h * 8 + d] = acc[h][d] * c;
+        }
+        float f2[N8 / 2];
+#pragma unroll
+        for (int i = 0; i < N8 / 2; i++) {
+            const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(f[i]), __float_as_uint(f[i + N8 / 2]), false, false);
+            f2[i] = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+        }
+#pragma unroll
+        for (int i = 0; i < N4; i++) {
+            const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(f2[i]), __float_as_uint(f2[i + N4]), false, false);
+            float v = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+            if constexpr (LPP <= 8) v += dpp_src<0x120 + (LPP <= 8 ? LPP : 1), 0xf>(v);      // row_ror:LPP
+            if constexpr (LPP <= 4) v += dpp_src<0x120 + (LPP <= 4 ? 2 * LPP : 1), 0xf>(v);  // row_ror:2 LPP
+            if constexpr (LPP <= 2) v += dpp_src<0x120 + (LPP <= 2 ? 4 * LPP : 1), 0xf>(v);  // row_ror:4 LPP
+            a4[i] = v;
         }
     }
-    __syncthreads();
-    for (int t = tid; t < NSL * G; t += kBlock) {
-        const int h = t / NSL, sl = t - h * NSL;
-        float M = -INFINITY;
-#pragma unroll 8
-        for (int i = 0; i < NSL; i++) M = fmaxf(M, s_m[i][h]);
-        s_c[sl][h] = M == -INFINITY ? 0.f : exp2_hw(s_m[sl][h] - M);
-        if (sl == 0) s_M[h] = M;
+    // The waves' sums meet in LDS: value i of a lane is number (lane >> 4's row quarter) * N4 + i of
+    // its G * 8, that is head (number / 8), dim lg * 8 + number % 8.
+    if ((lane & 15) < LPP) {
+        const int first = (lane >> 5) * (N8 / 2) + ((lane >> 4) & 1) * N4;
+#pragma unroll
+        for (int i = 0; i < N4; i += (N4 >= 4 ? 4 : 2)) {
+            const int v = first + i;
+            float* dst = &s_acc[wave][(v >> 3) * HD + lg * 8 + (v & 7)];
+            if constexpr (N4 >= 4)
+                *reinterpret_cast<float4*>(dst) = make_float4(a4[i], a4[i + 1], a4[i + 2], a4[i + 3]);
+            else
+                *reinterpret_cast<float2*>(dst) = make_float2(a4[i], a4[i + 1]);
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int h = 0; h < G; h++) {
+            s_m[wave][h] = m[h];
+            s_l[wave][h] = l[h];
+        }
     }
     __syncthreads();
 
@@ -399,13 +427,15 @@ __global__ __launch_bounds__(kBlock) void attn_split_kernel(const AttnParams p, 
     float* part = p.splits > 1 ? p.partials + (((size_t)b * p.nkv + g) * p.splits + split) * PS : nullptr;
     for (int idx = tid; idx < G * HD; idx += kBlock) {
         const int h = idx / HD, d = idx - h * HD;
-        const float M = s_M[h];
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) M = fmaxf(M, s_m[w][h]);
         float num = 0.f, den = 0.f;
-#pragma unroll 8
-        for (int i = 0; i < NSL; i++) {
-            const float c = s_c[i][h];
-            num = fmaf(c, s_acc[i][h][d], num);
-            den = fmaf(c, s_l[i][h], den);
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const float c = M == -INFINITY ? 0.f : exp2_hw(s_m[w][h] - M);
+            num = fmaf(c, s_acc[w][idx], num);
+            den = fmaf(c, s_l[w][h], den);
         }
         if (p.splits == 1) {
             if (h < gsize)
@@ -532,21 +562,21 @@ int launch_g(hipStream_t s, const AttnParams& p, int seq_len_step, size_t cache_
     // kernel; fp16 caches only (two steps of fp32 rows spill with eight heads). Measured on the 8B
     // shapes: 512 positions 8.9 -> 7.9 us at batch 1 and 10.5 -> 9.5 us at batch 8, 4096 positions
     // at batch 1 10.5 -> 9.5-9.8 us.
-    constexpr int kStep = (kWaves * 64 / (HD / 8)) * kUnroll;  // positions per step
+    constexpr int kSlots = kWaves * 64 / (HD / 8);  // position slots of a block
     constexpr bool SC = HD == 128 && G == 4;
-    bool short_slices = false;
-    if constexpr (CT == L0H_F16) {
-        short_slices = (int)ceil_div(p.max_seq_len, std::max(p.splits, 1)) <= 2 * kStep;
-        if (short_slices)
-            attn_split_kernel<HD, CT, QT, G, SC, true><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
-    }
-    if (!short_slices) {
-        const int per_split = p.max_seq_len / std::max(p.splits, 1);
-        if (SC && (per_split <= 256 || per_split >= 2048))
-            attn_split_kernel<HD, CT, QT, G, SC><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
-        else
-            attn_split_kernel<HD, CT, QT, G, false><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
-    }
+    const int per_split = (int)ceil_div(p.max_seq_len, std::max(p.splits, 1));
+    if (per_split <= kSlots)
+        attn_split_kernel<HD, CT, QT, G, 1, 1><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
+    else if (per_split <= 2 * kSlots)
+        attn_split_kernel<HD, CT, QT, G, 2, 1><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
+    else if (per_split <= kUnroll * kSlots)
+        attn_split_kernel<HD, CT, QT, G, kUnroll, 1, SC><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
+    else if (CT == L0H_F16 && per_split <= 2 * kUnroll * kSlots)
+        attn_split_kernel<HD, CT, QT, G, kUnroll, CT == L0H_F16 ? 2 : 0, SC><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
+    else if (SC && (per_split <= 256 || per_split >= 2048))
+        attn_split_kernel<HD, CT, QT, G, kUnroll, 0, SC><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
+    else
+        attn_split_kernel<HD, CT, QT, G, kUnroll, 0><<<grid, kBlock, 0, s>>>(p, seq_len_step, cache_batch_stride);
     int st = launch_status("attention");
     if (st || p.splits == 1) return st;
     constexpr int NC = G * HD / 4, CB = NC < 32 ? NC : 32;
@@ -1084,11 +1114,12 @@ int attention_default_splits(int batch, int nkv, int max_len, int compute_units)
     // x 32768 or batch 8 x 4096, 134 MB: 28.7 us against 33.7 us at two).
     // L0H_ATTN_SPLIT_POSITIONS overrides the minimum and L0H_ATTN_BLOCKS_PER_CU the blocks per CU
     // (tuning).
-    static const int min_pos = [] {
+    static const int min_env = [] {
         const char* e = std::getenv("L0H_ATTN_SPLIT_POSITIONS");
-        const int v = e ? std::atoi(e) : 128;
-        return v > 0 ? v : 128;
+        const int v = e ? std::atoi(e) : 0;
+        return v > 0 ? v : 0;
     }();
+    const int min_pos = min_env ? min_env : 128;
     static const int per_cu_env = [] {
         const char* e = std::getenv("L0H_ATTN_BLOCKS_PER_CU");
         const int v = e ? std::atoi(e) : 0;
@@ -1102,6 +1133,16 @@ int attention_default_splits(int batch, int nkv, int max_len, int compute_units)
         return std::max(1, std::min(kMaxSplits, std::min(target, by_len)));
     };
     if (per_cu_env) return splits_for(per_cu_env);
+    // Where slices of 64 positions make at most one block per CU, they are taken, up to the 64
+    // that the merge folds in one round: the kernel is then bound by the latency of one slice, not by
+    // bandwidth. One slice of up to 128 positions needs no merge and stays ahead. Measured (us, fp32 q,
+    // slices of 128 -> 64 -> 32 positions): 14 q / 2 kv heads of 64, 1000 positions fp32 10.0 -> 9.0 ->
+    // 8.7, 4000 10.7 -> 9.6 -> 10.6, fp16 142 9.2 -> 8.4 -> 8.5, 64 (one slice of 64, two of 32) 5.5 -> 8.5;
+    // 32 / 8 heads of 128, fp16 512 8.6 -> 7.8 -> 8.6, 2048 9.1 -> 8.6 -> 9.1;
+    // just past one block per CU, 2176 positions, 9.1 -> 9.5.
+    constexpr int kFine = 64;
+    const int fine = (len + kFine - 1) / kFine;
+    if (!min_env && fine > 2 && fine <= 64 && (long)batch * nkv * fine <= std::max(compute_units, 1)) return fine;
     const int two = splits_for(2);
     if (len / two >= 2048) return two;
     // Slices of four steps at one block per CU: twice the splits make them two-step slices, which
