@@ -1183,6 +1183,10 @@ int launch_attention_prefill(hipStream_t s, AttnParams p, int pos0, int tokens) 
             return fail(L0H_ERR_INVALID_ARG, "attention buffers must be 16-byte aligned");
         return p.head_dim == 64 ? launch_prefill_hd<64>(s, p, pos0, tokens) : launch_prefill_hd<128>(s, p, pos0, tokens);
     }
+    return launch_attention_tokens(s, p, pos0, tokens);
+}
+
+int launch_attention_tokens(hipStream_t s, AttnParams p, int pos0, int tokens) {
     p.batch = tokens;
     p.seq_len = pos0 + 1;
     p.seq_len_device = nullptr;

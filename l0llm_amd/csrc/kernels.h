@@ -84,8 +84,10 @@ struct GemvParams {
 int gemv_max_blocks(int compute_units, int per_cu = 2);
 
 int launch_gemv_nk(hipStream_t s, const GemvParams& p);
-// Up to 64 fp32 activation rows against int8, fp16 or bf16 weights (rows_kernel.h); the caller has
-// checked sizes and alignment (launch_gemv_nk).
+// Up to kGemvRowsMax fp32 activation rows against int8, fp16 or bf16 weights (rows_kernel.h), row m of
+// an EPI_QKV call at position pos0 + m; EPI_QKV and EPI_SWIGLU with norm_w, the others without. The
+// caller has checked sizes and alignment (as launch_gemv_nk does).
+constexpr int kGemvRowsMax = 64;
 int launch_gemv_rows(hipStream_t s, const GemvParams& p, int pos0);
 
 // Reference layout [K, N] GEMV / GEMM (Gemv.Execute, Gemm.Execute): rows in groups of up to 8,
@@ -161,6 +163,8 @@ int launch_attention_decode(hipStream_t s, const AttnParams& p);
 // Prefill over a shared cache: token t of the chunk attends to slots 0 .. pos0 + t (q and out
 // are [tokens, nh*hd]; p.batch and p.seq_len are set from pos0/tokens).
 int launch_attention_prefill(hipStream_t s, AttnParams p, int pos0, int tokens);
+// The same by the split decode kernel, token t of the chunk as batch entry t with length pos0 + t + 1.
+int launch_attention_tokens(hipStream_t s, AttnParams p, int pos0, int tokens);
 // True when the prefill runs the query-tiled kernel (no split workspace needed).
 bool attention_prefill_tiled(const AttnParams& p);
 

@@ -36,7 +36,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 rows_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float rows_f32x4;
 
 constexpr int kRowsStep = 64;        // K values per step
-constexpr int kRowsMax = 64;         // activation rows a launch takes
+constexpr int kRowsMax = kGemvRowsMax;
 constexpr int kRowsMaxK = 1 << 22;   // 64 rows of it stay under the 2 GiB of a buffer
 
 __device__ __forceinline__ rows_f32x4 rows_mfma(const uint4& a, const uint4& b, rows_f32x4 c) {
@@ -428,8 +428,11 @@ int dispatch_rows(hipStream_t s, const GemvParams& p, int pos0) {
     }
 }
 
+// The epilogues of a model's layer: q|k|v and gate|up take the norm with them, O and down none.
 template <int WT>
 int dispatch_rows_wt(hipStream_t s, const GemvParams& p, int pos0) {
+    if (p.epilogue == EPI_QKV) return dispatch_rows<WT, true, EPI_QKV>(s, p, pos0);
+    if (p.epilogue == EPI_SWIGLU) return dispatch_rows<WT, true, EPI_SWIGLU>(s, p, pos0);
     return dispatch_rows<WT, false, EPI_STORE>(s, p, pos0);
 }
 
