@@ -628,249 +628,190 @@ int launch_any(hipStream_t s, const AttnParams& p, int seq_len_step, size_t cach
 }
 
 // ---------------------------------------------------------------------------------------------
-// Causal prefill (Attention.ExecutePrefill, LlmDecoderLayer.cs:369-371), query-tiled: block
-// (query tile, kv head) holds 64 query vectors (64 / G tokens x the G q heads of the group) in LDS
-// and streams that kv head's K and V rows in tiles of 64 positions through LDS once for all of
-// them, so the cache is read once per tile of tokens instead of once per token. Scores, the online
-// softmax (fp32, log2 domain, as in the decode kernel) and P.V run on fp32 FMAs: thread
-// (ti, tj) = (tid / 16, tid % 16) owns query rows ti + 16 a and key columns tj + 16 b (a, b < 4),
-// and output dims 4 tj + 64 e; a row's 16 threads are 16 consecutive lanes, reduced by lane
-// shuffles. The next K/V tile is loaded into registers while the current one is computed; rows
-// past a query's position (and the tile padding) are clamped to valid cache rows and masked.
+// Causal prefill (Attention.ExecutePrefill, LlmDecoderLayer.cs:369-371) over an fp32 cache, fp32
+// throughout, on v_mfma_f32_16x16x4_f32. A query vector is a (token, q head of the group) pair; a block
+// holds 16 consecutive ones, in the registers of each of its four waves. A wave takes every fourth step
+// of 16 positions on its own, without LDS or barriers: a lane's operands are 16-byte pieces of the K and
+// V rows as they lie in memory. Scores, S^T = K Q^T: A is K (row = position l % 16), B is Q (column =
+// query l % 16), and the MFMA's k slot l / 16 stands for dim 16 s + 4 (l / 16) + j in product j of piece
+// s. Lane l then holds query l % 16 at the positions 4 (l / 16) + r. Product r of O^T += V^T P^T takes
+// exactly those: its k slot l / 16 is position 4 (l / 16) + r, B is P as it stands, and A is V's element
+// i of the lane's piece (dims 64 e + 4 (l % 16) + i), which makes the output's rows the dims of one i.
+// V is requested before the scores, the next K before the softmax; the waves' sums meet in LDS at the end.
+//
+// Bound by the fp32 MFMAs once the chip is full (32 q / 8 kv heads of 128, 2047 tokens: 34 GFLOP in
+// 371-400 us, 86-93 of 157 TFLOP/s), below that by the chain of one wave's steps. It took the place of fp32
+// FMAs on tiles in LDS (64 queries a block): that call 1491 -> 371-400 us, 14 / 2 heads of 64, 500 tokens
+// behind 37 64 -> 13 us, 14 tokens 10.3 -> 5.4. Four waves with different queries each, all steps of
+// them: 402, 28 and 5.0 us, and 463, 47 and 6.9 with 32 queries a wave (half the reads).
 // ---------------------------------------------------------------------------------------------
-constexpr int kPQ = 64;  // query vectors per block
-constexpr int kPK = 64;  // key positions per tile
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
-template <int HD>
-constexpr size_t prefill_smem_bytes() { return (size_t)(3 * 64 * (HD + 4) + 64 * (kPK + 4)) * sizeof(float); }
-
-__device__ __forceinline__ float row16_max(float v) {
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 16));
-    return v;
-}
-__device__ __forceinline__ float row16_sum(float v) {
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 16);
-    return v;
+// 4 consecutive query values (fp32 or fp16) as fp32.
+template <int QT>
+__device__ __forceinline__ f32x4_t load_q4(const void* base, size_t idx) {
+    if constexpr (QT == L0H_F32) {
+        return *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(base) + idx);
+    } else {
+        const uint2 a = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(base) + idx);
+        const float2 lo = __half22float2(__builtin_bit_cast(__half2, a.x)), hi = __half22float2(__builtin_bit_cast(__half2, a.y));
+        return f32x4_t{lo.x, lo.y, hi.x, hi.y};
+    }
 }
 
-template <int HD, int CT, int QT>
-__global__ __launch_bounds__(kBlock) void attn_prefill_tiled_kernel(const AttnParams p, int pos0, int tokens,
-                                                                    int gsize, int tq_tokens) {
-    extern __shared__ __attribute__((aligned(16))) float smem[];
-    constexpr int LD = HD + 4;     // row stride of the Q, K and V tiles (16-byte aligned rows)
-    constexpr int SLD = kPK + 4;   // row stride of the probability tile
-    constexpr int E = HD / 64;     // float4 output chunks per thread
-    constexpr int ES = CT == L0H_F16 ? 2 : 4;
-    constexpr int CPR = HD * ES / 16;            // 16-byte chunks per cache row
-    constexpr int NC = kPK * CPR / kBlock;       // chunks per thread per tile (K, and again V)
-    static_assert(NC >= 1 && (kPK * CPR) % kBlock == 0, "tile / block mismatch");
-    float* Qs = smem;
-    float* Ks = Qs + kPQ * LD;
-    float* Vs = Ks + kPK * LD;
-    float* Ps = Vs + kPK * LD;
+constexpr int kPrefillVec = 16;  // query vectors per block
 
-    const int tid = threadIdx.x, ti = tid >> 4, tj = tid & 15;
-    const int g = blockIdx.y;
-    // Query tiles in reverse: the last tokens see the most positions, so the longest blocks are
-    // dispatched first and the short ones fill in behind them.
-    const int t0 = (gridDim.x - 1 - blockIdx.x) * tq_tokens;
-    const int t_last = min(t0 + tq_tokens, tokens) - 1;
-    const int kmax = pos0 + t_last;  // last key position any query of the tile sees
+// Grid of the kernels whose blocks take `per` consecutive query vectors: kv head, then tile of vectors (the
+// kv head varies fastest: with 8 of them each XCD keeps one head's rows in its L2), and a block's tile, the
+// last first: those queries see the most positions, and the short blocks fill in behind them. Negative:
+// no tile (y x z rounds the count up; a grid's y is limited).
+constexpr int kTilesY = 32768;
+dim3 prefill_grid(int nkv, long nvec, int per) {
+    const long tiles = (nvec + per - 1) / per;
+    return dim3(nkv, (unsigned)std::min<long>(tiles, kTilesY), (unsigned)((tiles + kTilesY - 1) / kTilesY));
+}
+__device__ __forceinline__ int prefill_tile(int nvec, int per) {
+    return (nvec + per - 1) / per - 1 - (int)(blockIdx.z * gridDim.y + blockIdx.y);
+}
+
+template <int HD, int QT>
+__global__ __launch_bounds__(kBlock) void attn_prefill_f32_kernel(const AttnParams p, int pos0, int tokens, int gsize) {
+    constexpr int NS = HD / 16;  // 16-byte pieces of a K row per lane
+    constexpr int NE = HD / 64;  // 16-byte pieces of a V row per lane
+    __shared__ __attribute__((aligned(16))) float s_o[kWaves][kPrefillVec][HD + 4];
+    __shared__ float s_m[kWaves][kPrefillVec], s_l[kWaves][kPrefillVec];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lq = lane & 15, lg = lane >> 4;
+    const int g = blockIdx.x;
+    const int nvec = tokens * gsize;
+    const int v0 = prefill_tile(nvec, kPrefillVec) * kPrefillVec;
+    if (v0 < 0) return;
     const int row_elems = p.nkv * HD;
-    const typename CacheRow<CT>::T* kc = static_cast<const typename CacheRow<CT>::T*>(p.kc);
-    const typename CacheRow<CT>::T* vc = static_cast<const typename CacheRow<CT>::T*>(p.vc);
+    const float* kbase = static_cast<const float*>(p.kc) + (size_t)g * HD + 4 * lg;
+    const float* vbase = static_cast<const float*>(p.vc) + (size_t)g * HD + 4 * lq;
+    // Last position the block's first and last query see.
+    const int lim_first = pos0 + v0 / gsize;
+    const int kmax = pos0 + min(v0 + kPrefillVec - 1, nvec - 1) / gsize;
 
-    // Query vector i = token (t0 + i / gsize), head g * gsize + i % gsize; scaled by
-    // log2(e) / sqrt(HD). Vectors past the tile are zero and never written.
     const float qscale = 1.4426950408889634f / sqrtf((float)HD);
-    for (int c = tid; c < kPQ * (HD / 8); c += kBlock) {
-        const int i = c / (HD / 8), d = (c % (HD / 8)) * 8;
-        const int tq = i / gsize, t = t0 + tq;
-        float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (tq < tq_tokens && t < tokens) {
-            load8<QT>(p.q, (size_t)t * p.nh * HD + (size_t)(g * gsize + i % gsize) * HD + d, f);
+    f32x4_t q[NS];
+    const int vq = min(v0 + lq, nvec - 1), tq = vq / gsize, hq = g * gsize + vq - tq * gsize;
+    const int lim = pos0 + tq;  // (a lane past the last vector repeats it and stores nothing)
 #pragma unroll
-            for (int e = 0; e < 8; e++) f[e] *= qscale;
-        }
-        *reinterpret_cast<float4*>(&Qs[i * LD + d]) = make_float4(f[0], f[1], f[2], f[3]);
-        *reinterpret_cast<float4*>(&Qs[i * LD + d + 4]) = make_float4(f[4], f[5], f[6], f[7]);
-    }
-    // Last key position of each owned row (-1: padding row, fully masked).
-    int lim[4];
-#pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int i = ti + 16 * a, tq = i / gsize, t = t0 + tq;
-        lim[a] = (tq < tq_tokens && t < tokens) ? pos0 + t : -1;
-    }
+    for (int s = 0; s < NS; s++) q[s] = load_q4<QT>(p.q, ((size_t)tq * p.nh + hq) * HD + 16 * s + 4 * lg) * qscale;
 
-    // K / V tile kt into registers: chunk c of this thread is row (tid + c * kBlock) / CPR.
-    uint4 kr[NC], vr[NC];
-    auto load_tile = [&](int kt) {
+    f32x4_t kr[NS], vr[4][NE];
+    auto load_k = [&](int base) {
+        const float* r = kbase + (size_t)min(base + lq, kmax) * row_elems;
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const int q = tid + c * kBlock, r = q / CPR, col = q % CPR;
-            const int pos = min(kt * kPK + r, kmax);
-            const size_t off = (size_t)pos * row_elems + (size_t)g * HD + col * (16 / ES);
-            kr[c] = ld_nt16(kc + off);
-            vr[c] = ld_nt16(vc + off);
-        }
+        for (int s = 0; s < NS; s++) kr[s] = *reinterpret_cast<const f32x4_t*>(r + 16 * s);
     };
-    auto store_tile = [&]() {
+    auto load_v = [&](int base) {
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const int q = tid + c * kBlock, r = q / CPR, col = q % CPR;
-            float* kd = &Ks[r * LD + col * (16 / ES)];
-            float* vd = &Vs[r * LD + col * (16 / ES)];
-            if constexpr (CT == L0H_F16) {
-                const uint32_t kw[4] = {kr[c].x, kr[c].y, kr[c].z, kr[c].w};
-                const uint32_t vw[4] = {vr[c].x, vr[c].y, vr[c].z, vr[c].w};
+        for (int r = 0; r < 4; r++) {
+            const float* row = vbase + (size_t)min(base + 4 * lg + r, kmax) * row_elems;
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const float2 k0 = __half22float2(__builtin_bit_cast(__half2, kw[2 * j]));
-                    const float2 k1 = __half22float2(__builtin_bit_cast(__half2, kw[2 * j + 1]));
-                    const float2 v0 = __half22float2(__builtin_bit_cast(__half2, vw[2 * j]));
-                    const float2 v1 = __half22float2(__builtin_bit_cast(__half2, vw[2 * j + 1]));
-                    *reinterpret_cast<float4*>(kd + 4 * j) = make_float4(k0.x, k0.y, k1.x, k1.y);
-                    *reinterpret_cast<float4*>(vd + 4 * j) = make_float4(v0.x, v0.y, v1.x, v1.y);
-                }
-            } else {
-                *reinterpret_cast<uint4*>(kd) = kr[c];
-                *reinterpret_cast<uint4*>(vd) = vr[c];
-            }
+            for (int e = 0; e < NE; e++) vr[r][e] = *reinterpret_cast<const f32x4_t*>(row + 64 * e);
         }
     };
 
-    float m[4], l[4];
-    float4 o[4][E];
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o[NE][4];
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        m[a] = -INFINITY;
-        l[a] = 0.f;
+    for (int e = 0; e < NE; e++)
 #pragma unroll
-        for (int e = 0; e < E; e++) o[a][e] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int i = 0; i < 4; i++) o[e][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    constexpr int kStride = 16 * kWaves;
+    const int first = wave * 16;
+    if (first <= kmax) load_k(first);
+    for (int base = first; base <= kmax; base += kStride) {
+        load_v(base);
+        f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[s][j], q[s][j], st, 0, 0, 0);
+        load_k(base + kStride);  // past the end: clamped, not used
+        if (base + 15 > lim_first) {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (base + 4 * lg + r > lim) st[r] = -INFINITY;
+        }
+        const float mx = slot_reduce<16, true>(fmaxf(fmaxf(st[0], st[1]), fmaxf(st[2], st[3])));
+        const float mn = fmaxf(m, mx);
+        const float ref = mn == -INFINITY ? 0.f : mn;  // no position seen yet: keep zeros
+        if (__builtin_amdgcn_ballot_w64(mn > m)) {  // else every factor is 1
+            const float c = exp2_hw(m - ref);
+            l *= c;
+#pragma unroll
+            for (int e = 0; e < NE; e++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[e][i] *= c;
+            m = mn;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            st[r] = exp2_hw(st[r] - ref);
+            l += st[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int e = 0; e < NE; e++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[e][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[r][e][i], st[r], o[e][i], 0, 0, 0);
     }
 
-    const int ntiles = kmax / kPK + 1;
-    load_tile(0);
-    for (int kt = 0; kt < ntiles; kt++) {
-        __syncthreads();  // the previous tile's K, V and P are no longer read
-        store_tile();
-        if (kt + 1 < ntiles) load_tile(kt + 1);
-        __syncthreads();
-
-        // Scores of rows ti + 16 a against keys tj + 16 b.
-        float sc[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) sc[a][b] = 0.f;
-#pragma unroll 4
-        for (int d = 0; d < HD; d += 4) {
-            float4 qa[4], kb[4];
-#pragma unroll
-            for (int a = 0; a < 4; a++) qa[a] = *reinterpret_cast<const float4*>(&Qs[(ti + 16 * a) * LD + d]);
-#pragma unroll
-            for (int b = 0; b < 4; b++) kb[b] = *reinterpret_cast<const float4*>(&Ks[(tj + 16 * b) * LD + d]);
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    sc[a][b] = fmaf(qa[a].x, kb[b].x, sc[a][b]);
-                    sc[a][b] = fmaf(qa[a].y, kb[b].y, sc[a][b]);
-                    sc[a][b] = fmaf(qa[a].z, kb[b].z, sc[a][b]);
-                    sc[a][b] = fmaf(qa[a].w, kb[b].w, sc[a][b]);
-                }
-        }
-        // Online softmax per row; probabilities to LDS, accumulators rescaled.
-#pragma unroll
-        for (int a = 0; a < 4; a++) {
-            float mt = -INFINITY;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int pos = kt * kPK + tj + 16 * b;
-                if (pos > lim[a]) sc[a][b] = -INFINITY;
-                mt = fmaxf(mt, sc[a][b]);
-            }
-            const float mn = fmaxf(m[a], row16_max(mt));
-            const float corr = mn == -INFINITY ? 1.f : exp2_hw(m[a] - mn);  // 0 while m is -inf
-            float ps = 0.f;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const float pr = mn == -INFINITY ? 0.f : exp2_hw(sc[a][b] - mn);
-                Ps[(ti + 16 * a) * SLD + tj + 16 * b] = pr;
-                ps += pr;
-            }
-            l[a] = l[a] * corr + row16_sum(ps);
-            m[a] = mn;
-#pragma unroll
-            for (int e = 0; e < E; e++) {
-                o[a][e].x *= corr;
-                o[a][e].y *= corr;
-                o[a][e].z *= corr;
-                o[a][e].w *= corr;
-            }
-        }
-        __syncthreads();
-        // o[rows][dims 4 tj + 64 e ..] += P . V
-#pragma unroll 2
-        for (int j = 0; j < kPK; j += 4) {
-            float4 pa[4];
-#pragma unroll
-            for (int a = 0; a < 4; a++) pa[a] = *reinterpret_cast<const float4*>(&Ps[(ti + 16 * a) * SLD + j]);
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++) {
-#pragma unroll
-                for (int e = 0; e < E; e++) {
-                    const float4 v = *reinterpret_cast<const float4*>(&Vs[(j + jj) * LD + 4 * tj + 64 * e]);
-#pragma unroll
-                    for (int a = 0; a < 4; a++) {
-                        const float pv = jj == 0 ? pa[a].x : jj == 1 ? pa[a].y : jj == 2 ? pa[a].z : pa[a].w;
-                        o[a][e].x = fmaf(pv, v.x, o[a][e].x);
-                        o[a][e].y = fmaf(pv, v.y, o[a][e].y);
-                        o[a][e].z = fmaf(pv, v.z, o[a][e].z);
-                        o[a][e].w = fmaf(pv, v.w, o[a][e].w);
-                    }
-                }
-            }
-        }
+    // Lane l holds query l % 16, dims 64 e + 16 (l / 16) + 4 r + i; its l is the sum of its positions.
+    const float sum = slot_reduce<16, false>(l);
+    if (lg == 0) {
+        s_m[wave][lq] = m;
+        s_l[wave][lq] = sum;
     }
-
-    // out[token][head][d] = o / l
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        if (lim[a] < 0) continue;
-        const int i = ti + 16 * a, t = t0 + i / gsize, h = g * gsize + i % gsize;
-        const float inv = l[a] > 0.f ? 1.f / l[a] : 0.f;
+    for (int e = 0; e < NE; e++)
 #pragma unroll
-        for (int e = 0; e < E; e++) {
-            const size_t base = (size_t)t * p.nh * HD + (size_t)h * HD + 4 * tj + 64 * e;
-            store_act(p.out, p.out_dtype, base + 0, o[a][e].x * inv);
-            store_act(p.out, p.out_dtype, base + 1, o[a][e].y * inv);
-            store_act(p.out, p.out_dtype, base + 2, o[a][e].z * inv);
-            store_act(p.out, p.out_dtype, base + 3, o[a][e].w * inv);
+        for (int r = 0; r < 4; r++)
+            *reinterpret_cast<f32x4_t*>(&s_o[wave][lq][64 * e + 16 * lg + 4 * r]) =
+                f32x4_t{o[e][0][r], o[e][1][r], o[e][2][r], o[e][3][r]};
+    __syncthreads();
+    for (int idx = tid; idx < kPrefillVec * HD / 4; idx += kBlock) {
+        const int qi = idx / (HD / 4), d = (idx - qi * (HD / 4)) * 4, v = v0 + qi;
+        if (v >= nvec) continue;
+        float M = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) M = fmaxf(M, s_m[w][qi]);
+        f32x4_t num = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        float den = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            const float c = M == -INFINITY ? 0.f : exp2_hw(s_m[w][qi] - M);
+            num += c * *reinterpret_cast<const f32x4_t*>(&s_o[w][qi][d]);
+            den = fmaf(c, s_l[w][qi], den);
         }
+        const float inv = den > 0.f ? 1.f / den : 0.f;
+        const int t = v / gsize, h = g * gsize + v - t * gsize;
+        const size_t at = ((size_t)t * p.nh + h) * HD + d;
+#pragma unroll
+        for (int i = 0; i < 4; i++) store_act(p.out, p.out_dtype, at + i, num[i] * inv);
     }
 }
 
-template <int HD, int CT, int QT>
-int launch_prefill_tiled(hipStream_t s, const AttnParams& p, int pos0, int tokens) {
+template <int HD, int QT>
+int launch_prefill_f32(hipStream_t s, const AttnParams& p, int pos0, int tokens) {
     const int gsize = p.nh / p.nkv;
-    const int tq = kPQ / gsize;
-    const size_t smem = prefill_smem_bytes<HD>();
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&attn_prefill_tiled_kernel<HD, CT, QT>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (attr != hipSuccess) return fail(L0H_ERR_DEVICE, "prefill attention: LDS size attribute refused");
-    dim3 grid(ceil_div(tokens, tq), p.nkv);
-    attn_prefill_tiled_kernel<HD, CT, QT><<<grid, kBlock, smem, s>>>(p, pos0, tokens, gsize, tq);
-    return launch_status("attn_prefill_tiled");
+    const long nvec = (long)tokens * gsize;
+    attn_prefill_f32_kernel<HD, QT><<<prefill_grid(p.nkv, nvec, kPrefillVec), kBlock, 0, s>>>(p, pos0, tokens, gsize);
+    return launch_status("attn_prefill_f32");
 }
 
 // ---------------------------------------------------------------------------------------------
-// Causal prefill on MFMA (fp16 cache): the same block tiling as the fp32 kernel (64 query vectors
-// of one kv head, K / V tiles of 64 positions), with wave w owning query vectors 16 w .. 16 w + 15.
+// Causal prefill on MFMA (fp16 cache), query-tiled: a block holds 64 query vectors (64 / G tokens x the
+// G q heads of the group) and streams that kv head's K and V rows in tiles of 64 positions through LDS
+// once for all of them, wave w owning query vectors 16 w .. 16 w + 15.
 // Scores are computed transposed, S^T = K Q^T, with v_mfma_f32_16x16x32_f16 (K fragments from LDS,
 // the wave's Q fragments in registers, fp16, pre-scaled by log2(e) / sqrt(d)): lane l then holds,
 // for query l % 16, the 16 positions 16 j + 4 (l / 16) + r of the tile (j, r < 4). Those values,
@@ -880,8 +821,9 @@ int launch_prefill_tiled(hipStream_t s, const AttnParams& p, int pos0, int token
 // lane reads its V^T operand as two 8-byte runs. O^T accumulates in registers (dims 16 i + 4 g + r
 // of query l % 16). P is rounded to fp16 for the MFMA; the softmax sums stay fp32.
 // ---------------------------------------------------------------------------------------------
+constexpr int kPQ = 64;  // query vectors per block
+constexpr int kPK = 64;  // key positions per tile
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
-typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
     return (uint32_t)__half_as_ushort(__float2half_rn(a)) | ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
@@ -1097,11 +1039,11 @@ int launch_prefill_mfma(hipStream_t s, const AttnParams& p, int pos0, int tokens
 
 template <int HD>
 int launch_prefill_hd(hipStream_t s, const AttnParams& p, int pos0, int tokens) {
-    if (p.cache_dtype == L0H_F16)  // MFMA; an fp32 cache keeps the fp32 kernel
+    if (p.cache_dtype == L0H_F16)  // 16-bit operands; an fp32 cache keeps fp32 ones
         return p.q_dtype == L0H_F16 ? launch_prefill_mfma<HD, L0H_F16>(s, p, pos0, tokens)
                                     : launch_prefill_mfma<HD, L0H_F32>(s, p, pos0, tokens);
-    return p.q_dtype == L0H_F16 ? launch_prefill_tiled<HD, L0H_F32, L0H_F16>(s, p, pos0, tokens)
-                                : launch_prefill_tiled<HD, L0H_F32, L0H_F32>(s, p, pos0, tokens);
+    return p.q_dtype == L0H_F16 ? launch_prefill_f32<HD, L0H_F16>(s, p, pos0, tokens)
+                                : launch_prefill_f32<HD, L0H_F32>(s, p, pos0, tokens);
 }
 
 }  // namespace

@@ -864,7 +864,7 @@ constexpr int kShortAttention = 128;
 int short_chunk(l0h_model* m, const int* ids, int pos0, int T, bool head) {
     const auto& c = m->cfg;
     hipStream_t s = m->dev->stream;
-    const int H = c.hidden_size, I = c.intermediate_size;
+    const int H = c.hidden_size;
     int st = l0h_write(m->dev, m->pf_ids, 0, ids, (size_t)T * sizeof(int));
     if (st) return st;
     if ((st = launch_embedding(s, m->pf_ids, m->embedding, m->pf_hidden, H, (size_t)T * H))) return st;
