@@ -661,6 +661,20 @@ __device__ __forceinline__ f32x4_t load_q4(const void* base, size_t idx) {
 
 constexpr int kPrefillVec = 16;  // query vectors per block
 
+// Four consecutive outputs in one store (unaligned: `out` may start at any element).
+__device__ __forceinline__ void store_out4(const AttnParams& p, size_t at, f32x4_t v) {
+    typedef __attribute__((ext_vector_type(4), aligned(4))) float f32x4_u;
+    typedef __attribute__((ext_vector_type(4), aligned(2))) uint16_t u16x4_u;
+    if (p.out_dtype == L0H_F32) {
+        *reinterpret_cast<f32x4_u*>(static_cast<float*>(p.out) + at) = v;
+    } else {
+        u16x4_u b;
+#pragma unroll
+        for (int i = 0; i < 4; i++) b[i] = p.out_dtype == L0H_F16 ? __half_as_ushort(__float2half_rn(v[i])) : float_to_bf16_bits(v[i]);
+        *reinterpret_cast<u16x4_u*>(static_cast<uint16_t*>(p.out) + at) = b;
+    }
+}
+
 // Grid of the kernels whose blocks take `per` consecutive query vectors: kv head, then tile of vectors (the
 // kv head varies fastest: with 8 of them each XCD keeps one head's rows in its L2), and a block's tile, the
 // last first: those queries see the most positions, and the short blocks fill in behind them. Negative:
@@ -794,9 +808,7 @@ __global__ __launch_bounds__(kBlock) void attn_prefill_f32_kernel(const AttnPara
         }
         const float inv = den > 0.f ? 1.f / den : 0.f;
         const int t = v / gsize, h = g * gsize + v - t * gsize;
-        const size_t at = ((size_t)t * p.nh + h) * HD + d;
-#pragma unroll
-        for (int i = 0; i < 4; i++) store_act(p.out, p.out_dtype, at + i, num[i] * inv);
+        store_out4(p, ((size_t)t * p.nh + h) * HD + d, num * inv);
     }
 }
 
@@ -809,125 +821,119 @@ int launch_prefill_f32(hipStream_t s, const AttnParams& p, int pos0, int tokens)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Causal prefill on MFMA (fp16 cache), query-tiled: a block holds 64 query vectors (64 / G tokens x the
-// G q heads of the group) and streams that kv head's K and V rows in tiles of 64 positions through LDS
-// once for all of them, wave w owning query vectors 16 w .. 16 w + 15.
-// Scores are computed transposed, S^T = K Q^T, with v_mfma_f32_16x16x32_f16 (K fragments from LDS,
-// the wave's Q fragments in registers, fp16, pre-scaled by log2(e) / sqrt(d)): lane l then holds,
-// for query l % 16, the 16 positions 16 j + 4 (l / 16) + r of the tile (j, r < 4). Those values,
-// after the online softmax (fp32, the row spread over the 4 lanes l % 16 + 16 g), are exactly a
-// B operand of the P.V MFMA O^T += V^T P^T when its 32 K slots of a chunk c are the positions
-// 32 c + 4 g + e (e < 4) and 32 c + 16 + 4 g + (e - 4) — so V is staged transposed in LDS and each
-// lane reads its V^T operand as two 8-byte runs. O^T accumulates in registers (dims 16 i + 4 g + r
-// of query l % 16). P is rounded to fp16 for the MFMA; the softmax sums stay fp32.
+// Causal prefill on MFMA (fp16 cache), query-tiled: a block holds 32 NQ consecutive query vectors ((token, q
+// head of the group) pairs of one kv head) and streams that head's K and V rows in tiles of 64 positions
+// through LDS once for all of them. PS = 1: a wave owns 32 vectors; PS = 2: two waves share 32 vectors, one
+// takes the first half of every tile's positions and one the second, and their sums meet at the end.
+// Scores are computed transposed, S^T = K Q^T, with v_mfma_f32_32x32x16_f16 (K fragments from LDS, the
+// wave's Q fragments in registers, fp16, pre-scaled by log2(e) / sqrt(d)): lane l then holds, for query
+// l % 32, the positions 8 (r / 4) + 4 (l / 32) + r % 4 of 32 (r < 16). After the online softmax (fp32, the
+// row spread over 2 lanes, each with its own share of the sum) values r = 8 c .. 8 c + 7 are the B operand of
+// the P.V MFMA O^T += V^T P^T when its K slots are those positions; the A operand, four positions of one
+// dim twice, comes from the row-major V tile by transposed LDS reads (ds_read_b64_tr_b16). P is rounded to
+// fp16 for the MFMA; the softmax sums stay fp32.
+//
+// What bounds it: the vector instructions around the products (32 values a lane and tile: subtract, 2^x, add,
+// half a conversion, half a maximum) and the LDS reads, with two to three waves a SIMD to overlap them; at
+// the largest sizes the spread of the causal blocks. It took the place of 16 vectors a wave with
+// 16 x 16 x 32 products and V transposed in registers, where every wave read all of K and V from LDS for 16
+// vectors: 32 / 8 heads of 128, 2047 tokens 127 -> 67 us (34 GFLOP, 270 -> 510 TFLOP/s), 500 behind 1000
+// 45.3 -> 33.6, 8 tokens 5.9 -> 5.5 (8.3 with the outputs stored one by one: 64 of them a lane); 14 / 2 heads of
+// 64, 500 behind 37 13.3 -> 9.4, 14 tokens 5.2 -> 5.1; 32 / 8 of 64, 300 10.8 -> 7.2. Two tile buffers and one
+// barrier a tile: 2047 tokens 73 -> 83 us (half the blocks fit a CU).
 // ---------------------------------------------------------------------------------------------
-constexpr int kPQ = 64;  // query vectors per block
-constexpr int kPK = 64;  // key positions per tile
+constexpr int kPrefillGroup = 64;  // q heads per kv head, at most
+constexpr int kPK = 64;            // key positions per tile
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
+typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
+// Two fp32 values rounded to fp16 (to nearest), as one conversion.
 __device__ __forceinline__ uint32_t pack_half2(float a, float b) {
-    return (uint32_t)__half_as_ushort(__float2half_rn(a)) | ((uint32_t)__half_as_ushort(__float2half_rn(b)) << 16);
+    typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, f16x2_t));
 }
 
-template <int HD, int QT>
-__global__ __launch_bounds__(kBlock) void attn_prefill_mfma_kernel(const AttnParams p, int pos0, int tokens,
-                                                                   int gsize, int tq_tokens) {
-    constexpr int KLD = HD + 8;        // K tile row stride (halves): 16 rows hit distinct banks
-    constexpr int VLD = kPK + 4;       // V^T row stride (halves): 34 dwords, so the 16 rows of a P.V
-                                       // operand read, and the 8-byte runs of a store, spread over the banks
-    constexpr int CPR = HD / 8;        // 16-byte chunks per cache row
-    constexpr int PPI = 64 / CPR;      // V positions per wave load (quads of 4 positions x CPR columns)
-    constexpr int NC = kPK * CPR / kBlock;  // chunks per thread per tile (K, and again V)
-    constexpr int KS = HD / 32;        // MFMA K steps over the head dim
-    constexpr int NI = HD / 16;        // 16-dim output sub-tiles
-    static_assert(NC >= 1 && (kPK * CPR) % kBlock == 0, "tile / block mismatch");
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[kPK * KLD];
-    __shared__ __attribute__((aligned(16))) uint16_t Vt[HD * VLD];
+// prefill_tile in rounds of `round` tiles, every second one reversed: of the blocks a CU holds together,
+// `round` apart, the longer stands beside the shorter (32 / 8 heads of 128, 1500 tokens: 53.5 -> 48.0 us).
+__device__ __forceinline__ int prefill_tile_snake(int nvec, int per, int round) {
+    const int tiles = (nvec + per - 1) / per, t = (int)(blockIdx.z * gridDim.y + blockIdx.y);
+    if (t >= tiles) return -1;
+    const int r = t / round, at = t - r * round, size = min(round, tiles - r * round);
+    return tiles - 1 - (r * round + ((r & 1) ? size - 1 - at : at));
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int lq = lane & 15, lg = lane >> 4;
-    const int g = blockIdx.y;
-    // Query tiles in reverse: the last tokens see the most positions, so the longest blocks are
-    // dispatched first and the short ones fill in behind them.
-    const int t0 = (gridDim.x - 1 - blockIdx.x) * tq_tokens;
-    const int t_last = min(t0 + tq_tokens, tokens) - 1;
-    const int kmax = pos0 + t_last;
+template <int HD, int QT, int NQ, int PS>
+__global__ __launch_bounds__(64 * NQ * PS) void attn_prefill_mfma_kernel(const AttnParams p, int pos0, int tokens, int gsize, int round) {
+    constexpr int NW = NQ * PS;
+    constexpr int NJ = 2 / PS;    // 32-position halves of a tile per wave
+    constexpr int KLD = HD + 8;   // K tile row stride (halves): 16 rows hit distinct banks
+    constexpr int VLD = HD + 32;  // V tile row stride: rows 16 banks apart, 8 of them in a transposed read
+    constexpr int CPR = HD / 8;   // 16-byte chunks per cache row
+    constexpr int NC = CPR / NW;  // chunks per thread per tile (K, and again V)
+    constexpr int KS = HD / 16;   // MFMA K steps over the head dim
+    constexpr int NI = HD / 32;   // 32-dim output sub-tiles
+    __shared__ __attribute__((aligned(16))) uint16_t smem[kPK * (KLD + VLD)];  // a tile's K rows, then its V rows
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lq = lane & 31, lh = lane >> 5;
+    const int group = wave % NQ, j0 = wave / NQ;  // the wave's query vectors, and its half of a tile (PS = 2)
+    const int g = blockIdx.x;
+    const int nvec = tokens * gsize;
+    const int b0 = prefill_tile_snake(nvec, 32 * NQ, round) * (32 * NQ);
+    if (b0 < 0) return;
+    const int kmax = pos0 + min(b0 + 32 * NQ - 1, nvec - 1) / gsize;
     const int row_elems = p.nkv * HD;
-    const uint16_t* kc = static_cast<const uint16_t*>(p.kc);
-    const uint16_t* vc = static_cast<const uint16_t*>(p.vc);
+    const uint16_t* kc = static_cast<const uint16_t*>(p.kc) + (size_t)g * HD;
+    const uint16_t* vc = static_cast<const uint16_t*>(p.vc) + (size_t)g * HD;
 
-    // This lane's query vector: i = 16 wave + l % 16 -> token t0 + i / gsize, head g gsize + i % gsize.
-    const int qi = wave * 16 + lq;
-    const int qtok = qi / gsize;
-    const bool qvalid = qtok < tq_tokens && t0 + qtok < tokens;
-    const int lim = qvalid ? pos0 + t0 + qtok : -1;
-    const int lim_min = pos0 + t0;  // the last position the block's first query sees
+    // This lane's query vector (a lane past the last one repeats it and stores nothing), and the last
+    // positions the wave's first and last vectors see.
+    const int v = min(b0 + group * 32 + lq, nvec - 1), tq = v / gsize, hq = g * gsize + v - tq * gsize;
+    const int lim = pos0 + tq;
+    const int lim_first = pos0 + min(b0 + group * 32, nvec - 1) / gsize, lim_last = pos0 + min(b0 + group * 32 + 31, nvec - 1) / gsize;
     const float qscale = 1.4426950408889634f / sqrtf((float)HD);
-    uint4 qf[KS];  // Q[qi][32 kk + 8 lg .. +7] as fp16
+    uint4 qf[KS];  // dims 16 kk + 8 lh .. +7 as fp16
 #pragma unroll
     for (int kk = 0; kk < KS; kk++) {
-        float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (qvalid)
-            load8<QT>(p.q, (size_t)(t0 + qtok) * p.nh * HD + (size_t)(g * gsize + qi % gsize) * HD + 32 * kk + 8 * lg, f);
+        float f[8];
+        load8<QT>(p.q, ((size_t)tq * p.nh + hq) * HD + 16 * kk + 8 * lh, f);
         qf[kk] = make_uint4(pack_half2(f[0] * qscale, f[1] * qscale), pack_half2(f[2] * qscale, f[3] * qscale),
                             pack_half2(f[4] * qscale, f[5] * qscale), pack_half2(f[6] * qscale, f[7] * qscale));
     }
 
-    // Tile kt. K: chunk c of this thread is position (tid + c * kBlock) / CPR, dims
-    // 8 ((tid + c * kBlock) % CPR) (a wave reads whole rows). V: lane l of wave w holds, for chunk
-    // c, position 16 w + c PPI + 4 ((l / 4) / CPR) + l % 4 and dims 8 ((l / 4) % CPR) .. +7: the 4
-    // lanes of a quad hold 4 consecutive positions of one 16-byte column, which a 4 x 4 transpose
-    // across the quad turns into 8-byte runs of the transposed tile (4 positions of one dim).
     uint4 kr[NC], vr[NC];
-    const int vq = lane >> 2, vj = lane & 3;
-    const int vcol = vq % CPR, vrow0 = 16 * wave + 4 * (vq / CPR);  // + c PPI: first position of the quad
     auto load_tile = [&](int kt) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const int q = tid + c * kBlock, r = q / CPR, col = q % CPR;
-            const int pos = min(kt * kPK + r, kmax);
-            kr[c] = ld_nt16(kc + (size_t)pos * row_elems + (size_t)g * HD + col * 8);
-            const int vpos = min(kt * kPK + vrow0 + c * PPI + vj, kmax);
-            vr[c] = ld_nt16(vc + (size_t)vpos * row_elems + (size_t)g * HD + vcol * 8);
-        }
-    };
-    // Transpose step across lanes l and l ^ M of a quad (DPP quad_perm), on the 32-bit dim pairs
-    // k and k ^ M: a lane whose bit M differs from k's takes the partner's pair k ^ M.
-    auto quad_step = [&](uint32_t (&w)[4], auto mc) {
-        constexpr int M = decltype(mc)::value;
-        constexpr int CTRL = M == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2] / [2,3,0,1]
-        const bool upper = (vj & M) != 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (k & M) continue;
-            const uint32_t pa = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[k], CTRL, 0xf, 0xf, false);
-            const uint32_t pb = (uint32_t)__builtin_amdgcn_mov_dpp((int)w[k ^ M], CTRL, 0xf, 0xf, false);
-            const uint32_t a = w[k], b = w[k ^ M];
-            w[k] = upper ? pb : a;
-            w[k ^ M] = upper ? b : pa;
+            const int i = tid + c * 64 * NW, r = i / CPR, col = i % CPR;
+            const size_t at = (size_t)min(kt * kPK + r, kmax) * row_elems + col * 8;
+            kr[c] = *reinterpret_cast<const uint4*>(kc + at);
+            vr[c] = *reinterpret_cast<const uint4*>(vc + at);
         }
     };
     auto store_tile = [&]() {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const int q = tid + c * kBlock, r = q / CPR, col = q % CPR;
-            *reinterpret_cast<u32x4_t*>(&Ks[r * KLD + col * 8]) = u32x4_t{kr[c].x, kr[c].y, kr[c].z, kr[c].w};
-            // w[p] after the transpose: dims 8 vcol + 2 vj, + 1 of position vrow0 + c PPI + p.
-            uint32_t w[4] = {vr[c].x, vr[c].y, vr[c].z, vr[c].w};
-            quad_step(w, std::integral_constant<int, 2>{});
-            quad_step(w, std::integral_constant<int, 1>{});
-            const int d = 8 * vcol + 2 * vj, p0 = vrow0 + c * PPI;
-            *reinterpret_cast<u32x2_t*>(&Vt[d * VLD + p0]) =
-                u32x2_t{(w[0] & 0xFFFFu) | (w[1] << 16), (w[2] & 0xFFFFu) | (w[3] << 16)};
-            *reinterpret_cast<u32x2_t*>(&Vt[(d + 1) * VLD + p0]) =
-                u32x2_t{(w[0] >> 16) | (w[1] & 0xFFFF0000u), (w[2] >> 16) | (w[3] & 0xFFFF0000u)};
+            const int i = tid + c * 64 * NW, r = i / CPR, col = i % CPR;
+            *reinterpret_cast<u32x4_t*>(smem + r * KLD + col * 8) = u32x4_t{kr[c].x, kr[c].y, kr[c].z, kr[c].w};
+            *reinterpret_cast<u32x4_t*>(smem + kPK * KLD + r * VLD + col * 8) = u32x4_t{vr[c].x, vr[c].y, vr[c].z, vr[c].w};
         }
     };
+    // Four V values of one dim: with its 16 lanes' 8-byte reads of 4 rows x 16 dims, lane t at row t / 4,
+    // dims 4 (t % 4) .. + 3, lane t gets dim t of the four rows.
+    const int vrow = 4 * lh + ((lane >> 2) & 3), vdim = (lane & 16) + 4 * (lane & 3);
+    typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+    auto read_v = [&](const uint16_t* at) {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                             (__attribute__((address_space(3))) s16x4_t*)const_cast<uint16_t*>(at)));
+    };
 
-    float m = -INFINITY, l = 0.f;
-    f32x4_t o[NI];
+    float m = -INFINITY, l = 0.f;  // l: the lane's own positions
+    f32x16_t o[NI];
 #pragma unroll
-    for (int i = 0; i < NI; i++) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < NI; i++) o[i] = f32x16_t{};
 
     const int ntiles = kmax / kPK + 1;
     load_tile(0);
@@ -936,104 +942,121 @@ __global__ __launch_bounds__(kBlock) void attn_prefill_mfma_kernel(const AttnPar
         store_tile();
         if (kt + 1 < ntiles) load_tile(kt + 1);
         __syncthreads();
+        const int p0 = kt * kPK + 32 * NJ * j0;  // the wave's first position
+        if (p0 > lim_last) continue;             // none of its queries sees that far
+        const uint16_t* Ks = smem + 32 * NJ * j0 * KLD;
+        const uint16_t* Vs = smem + kPK * KLD + (32 * NJ * j0 + vrow) * VLD + vdim;
 
-        // S^T sub-tiles j: rows = positions 16 j .. 16 j + 15, columns = this wave's 16 queries.
-        f32x4_t st[4];
+        f32x16_t st[NJ];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            st[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NJ; j++) {
+            st[j] = f32x16_t{};
 #pragma unroll
             for (int kk = 0; kk < KS; kk++) {
-                const uint4 a = *reinterpret_cast<const uint4*>(&Ks[(16 * j + lq) * KLD + 32 * kk + 8 * lg]);
-                st[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                               __builtin_bit_cast(f16x8_t, qf[kk]), st[j], 0, 0, 0);
+                const uint4 a = *reinterpret_cast<const uint4*>(&Ks[(32 * j + lq) * KLD + 16 * kk + 8 * lh]);
+                st[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, qf[kk]), st[j], 0, 0, 0);
             }
         }
-        // Online softmax for query l % 16 over the tile's 64 positions (this lane: 16 of them).
-        // MASKED: the tile reaches past some query's last position (the diagonal tiles). Other
-        // tiles are whole for every query of the block, so no score is masked and the running
-        // maximum is finite after them (m = -inf only before the first tile, where exp2(-inf)
-        // = 0 scales the still-zero sums); the lanes of invalid queries compute values never stored.
-        uint32_t ph[4][2];  // P as fp16 pairs: sub-tile j, rows r = 0,1 and 2,3
-        auto softmax = [&](auto masked) {
-            constexpr bool MASKED = decltype(masked)::value;
-            float mt = -INFINITY;
+        if (p0 + 32 * NJ - 1 > lim_first) {  // the diagonal
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < NJ; j++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    if constexpr (MASKED) {
-                        const int pos = kt * kPK + 16 * j + 4 * lg + r;
-                        if (pos > lim) st[j][r] = -INFINITY;
-                    }
-                    mt = fmaxf(mt, st[j][r]);
-                }
-            mt = fmaxf(mt, __shfl_xor(mt, 16));
-            mt = fmaxf(mt, __shfl_xor(mt, 32));
-            const float mn = fmaxf(m, mt);
-            const float corr = MASKED && mn == -INFINITY ? 1.f : exp2_hw(m - mn);
-            float ps = 0.f;
+                for (int r = 0; r < 16; r++)
+                    if (p0 + 32 * j + 8 * (r >> 2) + 4 * lh + (r & 3) > lim) st[j][r] = -INFINITY;
+        }
+        float mt = st[0][0];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float pr[4];
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    pr[r] = MASKED && mn == -INFINITY ? 0.f : exp2_hw(st[j][r] - mn);
-                    ps += pr[r];
-                }
-                ph[j][0] = pack_half2(pr[0], pr[1]);
-                ph[j][1] = pack_half2(pr[2], pr[3]);
-            }
-            ps += __shfl_xor(ps, 16);
-            ps += __shfl_xor(ps, 32);
-            l = l * corr + ps;
+            for (int r = 0; r < 16; r++) mt = fmaxf(mt, st[j][r]);
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+        const float mn = fmaxf(m, fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])));
+        const float ref = mn == -INFINITY ? 0.f : mn;
+        if (__builtin_amdgcn_ballot_w64(mn > m)) {  // else every factor is 1
+            const float c = exp2_hw(m - ref);
+            l *= c;
+#pragma unroll
+            for (int i = 0; i < NI; i++) o[i] *= c;
             m = mn;
-#pragma unroll
-            for (int i = 0; i < NI; i++) {
-                o[i][0] *= corr;
-                o[i][1] *= corr;
-                o[i][2] *= corr;
-                o[i][3] *= corr;
-            }
-        };
-        if (kt * kPK + kPK - 1 <= lim_min)
-            softmax(std::false_type{});
-        else
-            softmax(std::true_type{});
-        // O^T[dims][q] += V^T[dims][pos] P^T[pos][q], chunks c of 32 positions.
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const uint4 b = make_uint4(ph[2 * c][0], ph[2 * c][1], ph[2 * c + 1][0], ph[2 * c + 1][1]);
-#pragma unroll
-            for (int i = 0; i < NI; i++) {
-                const uint16_t* vrow = &Vt[(16 * i + lq) * VLD + 32 * c + 4 * lg];
-                const uint2 lo = *reinterpret_cast<const uint2*>(vrow);
-                const uint2 hi = *reinterpret_cast<const uint2*>(vrow + 16);
-                const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
-                o[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a),
-                                                              __builtin_bit_cast(f16x8_t, b), o[i], 0, 0, 0);
-            }
         }
+        uint32_t ph[NJ][8];
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const float p0 = exp2_hw(st[j][r] - ref), p1 = exp2_hw(st[j][r + 1] - ref);
+                l += p0 + p1;
+                ph[j][r >> 1] = pack_half2(p0, p1);
+            }
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const uint4 b = make_uint4(ph[j][4 * c], ph[j][4 * c + 1], ph[j][4 * c + 2], ph[j][4 * c + 3]);
+#pragma unroll
+                for (int i = 0; i < NI; i++) {
+                    const uint16_t* at = Vs + (32 * j + 16 * c) * VLD + 32 * i;
+                    const uint2 lo = read_v(at), hi = read_v(at + 8 * VLD);
+                    o[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, make_uint4(lo.x, lo.y, hi.x, hi.y)),
+                                                                  __builtin_bit_cast(f16x8_t, b), o[i], 0, 0, 0);
+                }
+            }
     }
 
-    // out[token][head][16 i + 4 lg + r] = O^T / l for this lane's query.
-    if (qvalid) {
-        const int h = g * gsize + qi % gsize;
-        const float inv = l > 0.f ? 1.f / l : 0.f;
-        const size_t base = (size_t)(t0 + qtok) * p.nh * HD + (size_t)h * HD;
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    if constexpr (PS == 2) {  // the second half's sums join the first's, value by value of a lane
+        constexpr int NV = NI * 16 + 2;
+        static_assert(NQ * NV * 64 * 4 <= sizeof(smem), "the sums take the tile's place");
+        float* x = reinterpret_cast<float*>(smem) + group * NV * 64 + lane;
+        __syncthreads();
+        if (j0 == 1) {
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) x[(i * 16 + r) * 64] = o[i][r];
+            x[NI * 16 * 64] = m;
+            x[(NI * 16 + 1) * 64] = l;
+        }
+        __syncthreads();
+        if (j0 == 1) return;
+        const float m1 = x[NI * 16 * 64], M = fmaxf(m, m1);
+        const float c0 = m == -INFINITY ? 0.f : exp2_hw(m - M), c1 = m1 == -INFINITY ? 0.f : exp2_hw(m1 - M);
+        l = l * c0 + x[(NI * 16 + 1) * 64] * c1;
 #pragma unroll
         for (int i = 0; i < NI; i++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) store_act(p.out, p.out_dtype, base + 16 * i + 4 * lg + r, o[i][r] * inv);
+            for (int r = 0; r < 16; r++) o[i][r] = o[i][r] * c0 + x[(i * 16 + r) * 64] * c1;
+    }
+    if (b0 + group * 32 + lq < nvec) {
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+        const size_t base = ((size_t)tq * p.nh + hq) * HD + 4 * lh;
+#pragma unroll
+        for (int i = 0; i < NI; i++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+                store_out4(p, base + 32 * i + 2 * r, f32x4_t{o[i][r], o[i][r + 1], o[i][r + 2], o[i][r + 3]} * inv);
     }
 }
 
+// 32 vectors a block and two waves to share them while the chip has room for such blocks (64-vector ones
+// would leave CUs idle), then 64 vectors and two waves to each 32; at head_dim 128 from three 64-vector
+// blocks a CU on, one wave to each 32, which reads K and V once and not the sums twice. Measured (us, all
+// with outputs stored one by one; one wave / two on 32 vectors / two on 64): 14 / 2 heads of 64, 100 tokens
+// 6.6 / 6.0 / 6.6, 1000 19.9 / 16.1 / 15.9; 32 / 8 of 128, 250 13.0 / 11.8 / 12.7, 1000 32.6 / 31.2 / 28.5,
+// 1500 49.6 / 54.6 / 48.0, 1700 57.4 / 66.1 / 59.6; 32 / 8 of 64, 2047 42.0 / 45.4 / 38.4.
 template <int HD, int QT>
 int launch_prefill_mfma(hipStream_t s, const AttnParams& p, int pos0, int tokens) {
+    constexpr int kCus = 256;
     const int gsize = p.nh / p.nkv;
-    const int tq = kPQ / gsize;
-    dim3 grid(ceil_div(tokens, tq), p.nkv);
-    attn_prefill_mfma_kernel<HD, QT><<<grid, kBlock, 0, s>>>(p, pos0, tokens, gsize, tq);
+    const long nvec = (long)tokens * gsize, blocks = (nvec + 63) / 64 * p.nkv;
+    const int round = std::max(1, kCus / p.nkv);
+    if (blocks <= kCus)
+        attn_prefill_mfma_kernel<HD, QT, 1, 2><<<prefill_grid(p.nkv, nvec, 32), 128, 0, s>>>(p, pos0, tokens, gsize, round);
+    else if (HD == 128 && blocks >= 3 * kCus)
+        attn_prefill_mfma_kernel<HD, QT, 2, 1><<<prefill_grid(p.nkv, nvec, 64), 128, 0, s>>>(p, pos0, tokens, gsize, round);
+    else
+        attn_prefill_mfma_kernel<HD, QT, 2, 2><<<prefill_grid(p.nkv, nvec, 64), 256, 0, s>>>(p, pos0, tokens, gsize, round);
     return launch_status("attn_prefill_mfma");
 }
 
@@ -1111,7 +1134,7 @@ int launch_attention_decode(hipStream_t s, const AttnParams& p) {
 }
 
 bool attention_prefill_tiled(const AttnParams& p) {
-    return (p.head_dim == 64 || p.head_dim == 128) && p.nkv > 0 && p.nh % p.nkv == 0 && p.nh / p.nkv <= kPQ &&
+    return (p.head_dim == 64 || p.head_dim == 128) && p.nkv > 0 && p.nh % p.nkv == 0 && p.nh / p.nkv <= kPrefillGroup &&
            (p.cache_dtype == L0H_F16 || p.cache_dtype == L0H_F32) && (p.q_dtype == L0H_F16 || p.q_dtype == L0H_F32);
 }
 
