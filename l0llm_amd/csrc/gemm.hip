@@ -910,12 +910,33 @@ bool lds_plan_for(int dtype, int m, int n, int k, int cus, LdsPlan& out) {
     // meet once per two stages of a six-stage ring: Llama-3.2-1B bf16 q|k|v at M = 512 19.7 -> 18.4
     // us, gate|up at M = 128 24.3 -> 23.2 us (three interleaved runs each, cold weights).
     const LdsPlan narrow_plan{128, 64, 1, 0, 2, 2};
+    // One 128 x 64 block for most CUs (half of them, below 256 rows), where the plan above does not hold:
+    // int8 weights, and K too short for the two-group form. Up to 128 rows at any block count, above only
+    // while the blocks are about one a CU, and from 256 rows while K is short. Measured (us, gemm_nk_kernel
+    // or a split of larger tiles -> this): int8 100 rows 2048 -> 16384 26.4 -> 18.0, 896 -> 9728 15.2 -> 10.3,
+    // bf16 14.1 -> 9.2; int8 200 rows 4096 -> 6144 36.4 -> 28.7, 500 rows 2048 -> 3072 23.6 -> 17.0; the other
+    // side: 200 rows 2048 -> 16384 (512 blocks) 33.8 -> 37.6, 300 rows 4096 -> 6144 (288) 39.2 -> 52.6, 300 rows
+    // 4096 -> 4096 27.4 -> 28.5.
+    const size_t cu = (size_t)std::max(cus, 1), b128 = blocks(128, 64), b64 = blocks(64, 64);
+    const bool narrow_one = (dtype == L0H_I8PC || (m < 256 && k < 1024)) && b128 >= (m < 256 ? want * 2 / 3 : want) &&
+                            (m <= 128 || (m < 256 ? 4 * b128 <= 5 * cu : b128 <= cu && k <= 2560));
+    // 64 x 64 blocks, at most one a CU, where nothing larger fills the chip and K is short enough to take
+    // whole (with half a block per CU or fewer only up to 1024). Measured (us, as above): 896 -> 896 100 rows
+    // int8 9.4 -> 7.4, bf16 8.0 -> 6.8, 500 rows 9.9 -> 8.1; 300 rows 2048 -> 2048 17.2 -> 13.8 and 16.6 ->
+    // 11.6; 200 rows 2048 -> 2048 (128 blocks) 12.0 -> 13.5. Split over K it wins only a little (4864 -> 896,
+    // 300 rows 21.3 -> 18.4) and would ask calls for a larger workspace.
+    const bool square = m > 64 && k <= 2560 && b64 <= cu && (k <= 1024 || 2 * b64 > cu);
     if (m < 256) {
         if (narrow && m > 64 && k >= 1024) {
             out = narrow_plan;
             return true;
         }
-        return false;
+        if (m > 64 && narrow_one) {
+            out = LdsPlan{128, 64, 1};
+            return true;
+        }
+        if (square) out = LdsPlan{64, 64, 1};
+        return square;
     }
     static const bool big = [] {  // tuning: L0H_GEMM_LDS_256=0 keeps tall shapes on 128 x 256
         const char* e = std::getenv("L0H_GEMM_LDS_256");
@@ -934,6 +955,10 @@ bool lds_plan_for(int dtype, int m, int n, int k, int cus, LdsPlan& out) {
         }
     if (narrow) {
         out = narrow_plan;
+        return true;
+    }
+    if (narrow_one || square) {
+        out = narrow_one ? LdsPlan{128, 64, 1} : LdsPlan{64, 64, 1};
         return true;
     }
     for (int sp = 2; sp <= kMaxSplits && k / sp >= 8 * 64; sp *= 2)
