@@ -770,10 +770,10 @@ int run_step(l0h_model* m, int token, int position) {
 // ---- chunked prefill (LlmModel.Prefill, LlmModel.cs:320-385; LlmDecoderLayer.ForwardBatch,
 // LlmDecoderLayer.cs:337-378): the tokens of a chunk go through each layer together, their
 // projections as one MFMA GEMM (int8 / fp16 / bf16 weights, 64 rows or more; activations rounded
-// to fp16, or to bf16 for bf16 weights) or one multi-row GEMV (fp32 weights, short chunks: each
-// launch reads W once per 8 rows), their attention through the query-tiled causal kernel, and their k / v rows into the
+// to fp16, or to bf16 for bf16 weights) or one multi-row GEMV (fp32 weights, widths that are not a
+// multiple of 32; chunks of under 64 tokens go through short_chunk), their attention through the query-tiled causal kernel, and their k / v rows into the
 // cache. Only the cache carries a chunk's result forward, so the last layer stops after its
-// attention's cache writes. int8 weights go through the MFMA GEMM as well (exact int8 -> fp16
+// cache writes. int8 weights go through the MFMA GEMM as well (exact int8 -> fp16
 // in registers, fp16 activations, row scale in the epilogue): the multi-row GEMV would re-read a
 // wide-K matrix (down: K = 14336) once per token. Chunks of 2048 tokens: at the 8B shapes
 // 2048-token prefill takes 0.088 s in chunks of 256, 0.069 s in 512, 0.062 s in 1024 and 0.059 s
