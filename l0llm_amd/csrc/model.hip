@@ -771,8 +771,8 @@ int run_step(l0h_model* m, int token, int position) {
 // LlmDecoderLayer.cs:337-378): the tokens of a chunk go through each layer together, their
 // projections as one MFMA GEMM (int8 / fp16 / bf16 weights, 64 rows or more; activations rounded
 // to fp16, or to bf16 for bf16 weights) or one multi-row GEMV (fp32 weights, widths that are not a
-// multiple of 32; chunks of under 64 tokens go through short_chunk), their attention through the query-tiled causal kernel, and their k / v rows into the
-// cache. Only the cache carries a chunk's result forward, so the last layer stops after its
+// multiple of 32; chunks of under 64 tokens go through short_chunk), their attention through the
+// query-tiled causal kernel, and their k / v rows into the cache. Only the cache carries a chunk's result forward, so the last layer stops after its
 // cache writes. int8 weights go through the MFMA GEMM as well (exact int8 -> fp16
 // in registers, fp16 activations, row scale in the epilogue): the multi-row GEMV would re-read a
 // wide-K matrix (down: K = 14336) once per token. Chunks of 2048 tokens: at the 8B shapes
